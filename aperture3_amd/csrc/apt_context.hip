@@ -2410,7 +2410,7 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
       // 512, 70 with 2048; FP64 152, 140)
       cell_runs_shape(ctx->mesh, T, ctx->logsph ? 2048 : 512, ctx->runs);
       const uint64_t entries = cell_runs_size(ctx->mesh, ctx->runs);
-      HIPCHK(hipMalloc(&ctx->run_off, (entries + 1 + 2 * (uint64_t)ctx->runs.items) * 4));
+      HIPCHK(hipMalloc(&ctx->run_off, (entries + 2 + 2 * (uint64_t)ctx->runs.items) * 4));
       ctx->runs.off = ctx->run_off;
       ctx->runs.work = ctx->run_off + entries;
     }
@@ -2432,10 +2432,17 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
     }
     return APT_OK;
   }
-  unsigned long long kept = 0;
-  HIPCHK(hipMemcpyAsync(&kept, ctx->sortw.count, 8, hipMemcpyDeviceToHost,
-                        ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  uint64_t kept = 0;
+  if (by_runs) {  // the table's last entry, then the items and the slots in tiles
+    uint32_t h[3];
+    HIPCHK(hipMemcpyAsync(h, ctx->runs.work - 1, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    kept = h[0];
+    ctx->runs.guard_slots = kept - h[2];
+  } else {
+    HIPCHK(hipMemcpyAsync(&kept, ctx->sortw.count, 8, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+  }
   // the slots freed by the compaction become empty
   if (kept < n) {
     uint32_t *cell = ctx->prec == APT_PREC_FP64 ? ctx->p64.cell : ctx->p32.cell;

@@ -66,9 +66,10 @@ inline TileAxis make_tile_axis(int N, int nt) {
 // Runs of cell-ordered slots by tile (apt_runs.hpp).  off[row nt0 + tx] is the
 // first slot of the cells of mesh row `row` (y fastest, guard rows included)
 // from tile tx's first cell on; a row's guard cells in x belong to its first
-// and last tile.  The last entry (rows nt0) is `end`.  work: the number of work
-// items, then two words per item (tile, part | parts << 16): the tiles, those
-// with many particles in several parts.
+// and last tile.  The last entry (rows nt0) is `end`.  work, right behind it:
+// the number of work items, the slots in tiles (the others are in guard rows),
+// then two words per item (tile, part | parts << 16): the tiles, those with many
+// particles in several parts.
 struct CellRuns {
   const uint32_t *off = nullptr, *work = nullptr;
   TileAxis ax[3];
@@ -77,8 +78,9 @@ struct CellRuns {
   uint32_t items;  // most items there can be (a multiple of 8)
   uint32_t least;  // particles below which a tile is not shared
   uint64_t end;    // slots covered, known on the host
+  uint64_t guard_slots;  // of these in guard rows (host counts)
 };
-// entries of the offsets; the table has 1 + 2 items more
+// entries of the offsets; the table has 2 + 2 items more
 inline uint64_t cell_runs_size(const Mesh &m, const CellRuns &cr) {
   return (uint64_t)m.dims[1] * m.dims[2] * cr.nt[0] + 1;
 }

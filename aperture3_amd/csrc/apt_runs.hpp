@@ -43,15 +43,33 @@ __device__ __forceinline__ int fold_axis(const Mesh &m, int ax, int i) {
   return g + r;
 }
 
+// f(slot) for every slot that the table holds in guard rows, a row a workgroup
+// at a time, a slot a lane.
+template <class F>
+__device__ __forceinline__ void for_guard_row_slots(const Mesh &m, const CellRuns &cr, const F &f) {
+  const uint32_t rows = (uint32_t)m.dims[1] * (uint32_t)m.dims[2];
+  for (uint32_t r = blockIdx.x; r < rows; r += gridDim.x) {
+    const int j = (int)(r % (uint32_t)m.dims[1]), k = (int)(r / (uint32_t)m.dims[1]);
+    if (m.in_bulk(m.guard[0], j, k)) continue;
+    const uint64_t e = (uint64_t)r * (uint64_t)cr.nt[0];
+    const uint32_t end = cr.off[e + (uint64_t)cr.nt[0]];
+    for (uint32_t i = cr.off[e] + threadIdx.x; i < end; i += blockDim.x) f(i);
+  }
+}
+inline unsigned guard_row_blocks(const Mesh &m) {
+  const uint64_t rows = (uint64_t)m.dims[1] * m.dims[2];
+  return (unsigned)(rows < 4096 ? rows : 4096);
+}
+
 // Work item of workgroup b: the items in use are spread over the XCDs as in
 // xcd_tile.  False: there is none.
 __device__ __forceinline__ bool run_item(const CellRuns &cr, uint32_t b, uint32_t &tile,
                                          uint32_t &part, uint32_t &parts) {
   const uint32_t n = cr.work[0], per = (n + 7u) >> 3, i = (b & 7u) * per + (b >> 3);
   if ((b >> 3) >= per || i >= n) return false;
-  tile = cr.work[1 + 2 * i];
-  part = cr.work[2 + 2 * i] & 0xffffu;
-  parts = cr.work[2 + 2 * i] >> 16;
+  tile = cr.work[2 + 2 * i];
+  part = cr.work[3 + 2 * i] & 0xffffu;
+  parts = cr.work[3 + 2 * i] >> 16;
   return true;
 }
 

@@ -820,8 +820,8 @@ void f64_runs_tile(int dim, int T[3]) {
 // spread over the share, so neighbouring lanes read whole cache lines while
 // the wave's atomics fall on many cells; in 1D, where a tile is a few cells
 // wide, lanes also alternate between copies of the window.  Particles outside
-// the window deposit straight to HBM (counted).  Workgroups past the tiles
-// erase the slots of guard rows.
+// the window deposit straight to HBM (counted).  The slots of guard rows are
+// k_push_guard_rows_f64's.
 template <int DIM, bool RHO>
 __attribute__((amdgpu_waves_per_eu(F64RunShape<DIM>::WAVES))) __global__ void
     __launch_bounds__(F64RunShape<DIM>::NT) k_push_deposit_f64_runs(Mesh m, Species sp, double dt, int H, PtcF64 p, FieldsF64 f, AccF64 a,
@@ -842,18 +842,6 @@ __attribute__((amdgpu_waves_per_eu(F64RunShape<DIM>::WAVES))) __global__ void
   __shared__ long long *s_dst[14];
   __shared__ double s_qdt[8], s_q[8];  // dt q / 2m and q per species
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const uint32_t nwork = cr.items;
-  if (blockIdx.x >= nwork) {
-    const uint64_t rows = (uint64_t)m.dims[1] * m.dims[2];
-    for (uint64_t r = (uint64_t)(blockIdx.x - nwork) * NT + tid; r < rows;
-         r += (uint64_t)(gridDim.x - nwork) * NT) {
-      const int j = (int)(r % (uint64_t)m.dims[1]), k = (int)(r / (uint64_t)m.dims[1]);
-      if (m.in_bulk(m.guard[0], j, k)) continue;
-      for (uint32_t i = cr.off[r * cr.nt[0]]; i < cr.off[(r + 1) * cr.nt[0]]; i++)
-        p.cell[i] = MAX_CELL;
-    }
-    return;
-  }
   uint32_t tile, part, parts;
   if (!run_item(cr, blockIdx.x, tile, part, parts)) return;  // uniform
   for (int e = tid; e < NC * 2 * NQ * WN; e += NT) win[e] = 0;
@@ -1002,6 +990,29 @@ __attribute__((amdgpu_waves_per_eu(F64RunShape<DIM>::WAVES))) __global__ void
   }
 }
 
+// The slots that a sort left in guard rows, which belong to no tile (none on a
+// periodic mesh: not launched then).  Each is judged by its own cell, not by the
+// row it was sorted into: a recorded step may be replayed on particles that were
+// set since.
+template <int DIM>
+__global__ void __launch_bounds__(64)
+    k_push_guard_rows_f64(Mesh m, Species sp, double dt, int H, int rho, PtcF64 p, FieldsF64 f,
+                          AccF64 a, CellRuns cr, unsigned long long *__restrict__ counters) {
+  for_guard_row_slots(m, cr, [&](uint32_t idx) {
+    const uint32_t c = p.cell[idx];
+    if (c == MAX_CELL) return;
+    int c1, c2, c3;
+    m.split(c, c1, c2, c3);
+    if (!m.in_bulk(c1, c2, c3)) {
+      p.cell[idx] = MAX_CELL;
+      return;
+    }
+    push_deposit_f64<DIM>(m, sp, dt, rho, p, f, counters, idx, c1, c2, c3,
+                          DepGlobal{m, a, H, c1, c2, c3});
+    atomicAdd(&counters[CTR_GLOBAL_DEP], 1ull);
+  });
+}
+
 // J = hi 2^-H + lo 2^-(H+40), accumulators cleared for the next step.
 __global__ void k_finalize_f64(long long *__restrict__ hi,
                                long long *__restrict__ lo,
@@ -1052,10 +1063,17 @@ hipError_t launch_push_deposit_f64_runs(const Mesh &m, const Species &sp, double
   Species spd = sp;
   for (int i = 0; i < 8; i++) spd.qdt[i] = dt * 0.5 * sp.q[i] / sp.m[i];
   auto go = [&](auto kern, int NT) {
-    const uint32_t extra = m.dims[1] * m.dims[2] > m.N[1] * m.N[2] ? 1 : 0;  // guard rows
-    kern<<<(unsigned)(cr.items + extra), NT, 0, st>>>(m, spd, dt, H, p, f, a, cr, counters);
+    kern<<<cr.items, NT, 0, st>>>(m, spd, dt, H, p, f, a, cr, counters);
     return hipGetLastError();
   };
+  if (cr.guard_slots > 0 && m.dim > 1) {
+    if (m.dim == 2)
+      k_push_guard_rows_f64<2><<<guard_row_blocks(m), 64, 0, st>>>(m, spd, dt, H, rho, p, f, a, cr,
+                                                                   counters);
+    else
+      k_push_guard_rows_f64<3><<<guard_row_blocks(m), 64, 0, st>>>(m, spd, dt, H, rho, p, f, a, cr,
+                                                                   counters);
+  }
   if (m.dim == 1)
     return rho ? go(k_push_deposit_f64_runs<1, true>, F64RunShape<1>::NT)
                : go(k_push_deposit_f64_runs<1, false>, F64RunShape<1>::NT);

@@ -257,18 +257,6 @@ __global__ void __launch_bounds__(MixedRunShape<DIM>::NT)
   __shared__ unsigned long long win[NC * NQ * WN];
   __shared__ RunWalk<S::T1 * S::T2> walk;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const uint32_t nwork = cr.items;
-  if (blockIdx.x >= nwork) {  // the slots of guard rows
-    const uint64_t rows = (uint64_t)m.dims[1] * m.dims[2];
-    for (uint64_t r = (uint64_t)(blockIdx.x - nwork) * NT + tid; r < rows;
-         r += (uint64_t)(gridDim.x - nwork) * NT) {
-      const int j = (int)(r % (uint64_t)m.dims[1]), k = (int)(r / (uint64_t)m.dims[1]);
-      if (m.in_bulk(m.guard[0], j, k)) continue;
-      for (uint32_t i = cr.off[r * cr.nt[0]]; i < cr.off[(r + 1) * cr.nt[0]]; i++)
-        p.cell[i] = MAX_CELL;
-    }
-    return;
-  }
   uint32_t tile, part, parts;
   if (!run_item(cr, blockIdx.x, tile, part, parts)) return;  // uniform
   for (int e = tid; e < NC * NQ * WN; e += NT) win[e] = 0;
@@ -328,6 +316,29 @@ __global__ void __launch_bounds__(MixedRunShape<DIM>::NT)
   }
 }
 
+// The slots that a sort left in guard rows, which belong to no tile (see
+// k_push_guard_rows_f64).
+template <int DIM>
+__global__ void __launch_bounds__(64)
+    k_push_guard_rows_mixed(Mesh m, Species sp, float dt, float scale, PtcF32 p, FieldsF32 f,
+                            AccMixed a, CellRuns cr, unsigned long long *__restrict__ counters) {
+  for_guard_row_slots(m, cr, [&](uint32_t idx) {
+    const uint32_t c = p.cell[idx];
+    if (c == MAX_CELL) return;
+    int c1, c2, c3;
+    m.split(c, c1, c2, c3);
+    if (!m.in_bulk(c1, c2, c3)) {
+      p.cell[idx] = MAX_CELL;
+      return;
+    }
+    push_deposit_mixed<DIM>(m, sp, dt, a.rho, p, f, counters, idx, c1, c2, c3,
+                            [&](int q, int di, int dj, int dk, float v) {
+                              acc_fx(q < 3 ? a.J[q] : a.R[q - 3],
+                                     m.widx(c1 + di, c2 + dj, c3 + dk), v, scale);
+                            });
+  });
+}
+
 hipError_t launch_push_deposit_mixed_runs(const Mesh &m, const Species &sp, float dt, int S,
                                           const PtcF32 &p, const FieldsF32 &f, const AccMixed &a,
                                           const CellRuns &cr, unsigned long long *counters,
@@ -335,10 +346,17 @@ hipError_t launch_push_deposit_mixed_runs(const Mesh &m, const Species &sp, floa
   if (cr.end == 0) return hipSuccess;
   const float scale = ldexpf(1.0f, S);
   auto go = [&](auto kern, int NT) {
-    const uint32_t extra = m.dims[1] * m.dims[2] > m.N[1] * m.N[2] ? 1 : 0;  // guard rows
-    kern<<<cr.items + extra, NT, 0, st>>>(m, sp, dt, scale, p, f, a, cr, counters);
+    kern<<<cr.items, NT, 0, st>>>(m, sp, dt, scale, p, f, a, cr, counters);
     return hipGetLastError();
   };
+  if (cr.guard_slots > 0 && m.dim > 1) {
+    if (m.dim == 2)
+      k_push_guard_rows_mixed<2><<<guard_row_blocks(m), 64, 0, st>>>(m, sp, dt, scale, p, f, a, cr,
+                                                                     counters);
+    else
+      k_push_guard_rows_mixed<3><<<guard_row_blocks(m), 64, 0, st>>>(m, sp, dt, scale, p, f, a, cr,
+                                                                     counters);
+  }
   if (m.dim == 1) return go(k_push_deposit_mixed_runs<1>, MixedRunShape<1>::NT);
   if (m.dim == 2) return go(k_push_deposit_mixed_runs<2>, MixedRunShape<2>::NT);
   return go(k_push_deposit_mixed_runs<3>, MixedRunShape<3>::NT);

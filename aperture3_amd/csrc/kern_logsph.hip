@@ -545,20 +545,25 @@ __global__ void __launch_bounds__(LS_NT, (ls_waves<R, RHO>()))
     cnt = hi - lo;
     x0 = org[0] - LS_HALO;
     y0 = org[1] - LS_HALO;
-  } else if (nwork > 0 && blockIdx.x == nwork) {  // the slots of guard rows
-    for (int j = tid; j < m.dims[1]; j += LS_NT) {
-      if (j >= m.guard[1] && j < m.dims[1] - m.guard[1]) continue;
-      const uint64_t e = (uint64_t)j * cr.nt[0];
-      for (uint32_t i = cr.off[e]; i < cr.off[e + cr.nt[0]]; i++) p.cell[i] = MAX_CELL;
-    }
-    return;
   } else {
+    // The slots that no tile holds: one workgroup takes those sorted into the
+    // guard rows below the tiles, the others those above them, which end where
+    // the slots behind the sorted ones begin.  Each is judged by its own cell, as
+    // a recorded step may be replayed on particles that were set since the sort.
     n = dev_n(n, dn);
-    const uint32_t first = nwork > 0 ? nwork + 1 : 0;
-    const uint64_t from = nwork > 0 ? cr.off[(uint64_t)m.dims[1] * m.dims[2] * cr.nt[0]] : 0;
+    const bool lower = nwork > 0 && blockIdx.x == nwork;  // uniform
+    const uint32_t first = lower ? nwork : nwork > 0 ? nwork + 1 : 0;
+    uint64_t from = 0, groups = 1;
+    if (lower) {
+      const uint64_t end = cr.off[(uint64_t)m.guard[1] * cr.nt[0]];
+      n = end < n ? end : n;
+    } else {
+      if (nwork > 0) from = cr.off[(uint64_t)(m.dims[1] - m.guard[1]) * cr.nt[0]];
+      groups = gridDim.x - first;
+    }
     if (from >= n) return;  // uniform
     // whole slots a thread: one, unless the grid is capped
-    const uint64_t per = (uint64_t)(gridDim.x - first) * LS_NT;
+    const uint64_t per = groups * LS_NT;
     const uint64_t chunk = (n - from + per - 1) / per * LS_NT;
     base = from + (uint64_t)(blockIdx.x - first) * chunk;
     if (base >= n) return;  // uniform: past the count
@@ -1277,6 +1282,7 @@ static hipError_t launch_logsph_push(const Mesh &m, const Species &sp, const LsP
   // of LDS while it finds out: 1024 x 1024 with
   // pairs, 0.42 -> 0.32 ms a push
   if (dn && tail > LS_DEV_TAIL) tail = LS_DEV_TAIL;
+  if (tail == 0) tail = 1;  // the guard rows above the tiles
   const uint64_t grid = nwork + (runs ? 1 : 0) + tail;
   const CellRuns cr = runs ? *runs : CellRuns{};
   if (rho)

@@ -92,12 +92,13 @@ __global__ void k_cell_runs(Mesh m, CellRuns cr, const uint32_t *__restrict__ ke
 // in tile order, 1024 tiles at a time.
 __global__ void __launch_bounds__(1024)
     k_cell_work(Mesh m, CellRuns cr, uint64_t per, uint32_t *__restrict__ work) {
-  __shared__ uint32_t s_w[16];
+  __shared__ uint32_t s_w[16], s_n;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  uint32_t base = 0;
+  uint32_t base = 0, mine = 0;
+  if (tid == 0) s_n = 0;
   for (uint32_t t0 = 0; t0 < cr.ntiles; t0 += 1024) {
     const uint32_t t = t0 + (uint32_t)tid;
-    uint32_t parts = 0;
+    uint32_t parts = 0, slots = 0;
     if (t < cr.ntiles) {
       const uint32_t tx = t % (uint32_t)cr.nt[0], r = t / (uint32_t)cr.nt[0];
       const int ty = (int)(r % (uint32_t)cr.nt[1]), tz = (int)(r / (uint32_t)cr.nt[1]);
@@ -110,7 +111,9 @@ __global__ void __launch_bounds__(1024)
         }
       const uint64_t q = (5 * n + 3 * per) / (5 * per);
       parts = n == 0 ? 0u : q < 1 ? 1u : q > 0xffff ? 0xffffu : (uint32_t)q;
+      slots = (uint32_t)n;
     }
+    mine += slots;
     uint32_t s = parts;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -125,12 +128,17 @@ __global__ void __launch_bounds__(1024)
       base += s_w[k];
     }
     for (uint32_t k = 0; k < parts; k++) {
-      work[1 + 2 * (at + k)] = t;
-      work[2 + 2 * (at + k)] = k | parts << 16;
+      work[2 + 2 * (at + k)] = t;
+      work[3 + 2 * (at + k)] = k | parts << 16;
     }
     __syncthreads();  // s_w is written again
   }
-  if (tid == 0) work[0] = base;
+  if (mine) atomicAdd(&s_n, mine);
+  __syncthreads();
+  if (tid == 0) {
+    work[0] = base;
+    work[1] = s_n;
+  }
 }
 
 // particles of a part: enough parts for about four workgroups per CU where
@@ -150,7 +158,7 @@ void cell_runs_shape(const Mesh &m, const int T[3], uint32_t least, CellRuns &cr
     cr.ntiles *= (uint32_t)cr.nt[d];
   }
   cr.items = (cr.ntiles + (cr.ntiles > RUN_WGS ? cr.ntiles : RUN_WGS) + 7u) / 8u * 8u;
-  cr.end = 0;
+  cr.end = cr.guard_slots = 0;
 }
 
 static inline unsigned blocks_for(uint64_t n) {
