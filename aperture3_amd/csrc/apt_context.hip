@@ -1793,8 +1793,12 @@ apt_status apt_ptc_update(apt_ctx *ctx, double dt, uint32_t step) {
     }
     if (ctx->mesh.dim == 3 && ctx->tiles_valid && !ctx->capturing) {
       const int iv = ctx->params.cell_order_interval == 0 ? 5 : ctx->params.cell_order_interval;
+      // a re-layout drops a recorded step; where an axis is no multiple of the
+      // tile extent it waits for the recording to go instead
+      bool ragged = false;
+      for (int d = 0; d < 3; d++) ragged = ragged || ctx->mesh.N[d] % ctx->tiles.T[d] != 0;
       if (iv > 0 && ctx->pushes_since_sort > 0 && ctx->pushes_since_sort % (uint32_t)iv == 0 &&
-          tile_cellsort_supported(ctx->tiles)) {
+          tile_cellsort_supported(ctx->tiles) && !(ragged && ctx->gexec)) {
         apt_status st = relayout_tiles(ctx);
         if (st != APT_OK) return st;
       }

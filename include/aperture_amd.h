@@ -401,7 +401,9 @@ apt_status apt_get_events(apt_ctx *ctx, uint64_t *emitted, uint64_t *converted,
  * (the charge-deposit cadence), time and dt, and the particle buffers of
  * the current sort parity (record again after a sort).  In a 3D tiled
  * mixed run an eager push that lays the tiles out again by cell (see
- * cell_order_interval) swaps those buffers and drops the recording. */
+ * cell_order_interval) swaps those buffers and drops the recording; on a
+ * mesh with an axis that is no multiple of the tile extent the tiles are
+ * not laid out again while there is a recording. */
 apt_status apt_graph_begin(apt_ctx *ctx);
 apt_status apt_graph_end(apt_ctx *ctx);
 apt_status apt_graph_launch(apt_ctx *ctx, int times);

@@ -95,3 +95,34 @@ def test_replay_of_a_log_spherical_step(precision, device):
                 pu.update_particles(d, c.dt, 0)
         out.append(d)
     check(*out)
+
+
+def test_recording_outlives_eager_pushes_on_a_ragged_3d_mesh():
+    """More eager pushes than a re-layout interval between recording and replay:
+    the recording is still there, and fields equal those of eager pushes alone."""
+    c = Case((12, 11, 9), 3, theta=(0.1, 0.1), drift=(0.2, -0.2), Bbg=(0.3, 0.0, 1.0))
+    state = c.oracle().particles()
+    out = []
+    for graph in (True, False):
+        env, d = c.gpu(precision=apt.APT_PREC_MIXED, load=False)
+        d.set_particles(state)
+        d.sort_particles()
+        pu, fs = apt.ptc_updater(env), apt.field_solver(env)
+
+        def step():
+            pu.update_particles(d, c.dt, 0)
+            fs.update_fields(d, c.dt, 1)
+
+        if graph:
+            d.graph_begin()
+            step()
+            d.graph_end()
+        for k in range(12):
+            if graph and k >= 8:
+                d.graph_launch(1)
+            else:
+                step()
+        out.append([d.get_field(w, q) for w in (apt.FIELD_E, apt.FIELD_B, apt.FIELD_J)
+                    for q in range(3)])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
