@@ -1,0 +1,68 @@
+"""The tables of the updates over runs of sorted slots on meshes of many tiles:
+more than one workgroup of work items, tiles that hold most of the particles and
+are shared, tiles that are empty.  FP64 against the oracle bit for bit; mixed
+against a context that is given the sorted particles and never sorts."""
+import numpy as np
+import pytest
+
+import aperture3_amd as apt
+from cases import Case
+from test_gpu_f64_runs import assert_same_fields
+from test_gpu_parity_cart import assert_same_particles, run_both
+
+pytestmark = pytest.mark.gpu
+
+# 1D: 563 tiles of 16 cells; 2D: 325; 3D: 8 x 4 x 4 FP64, 8^3 mixed: 780, 120
+MESHES = [(9000,), (200, 390), (43, 41, 50)]
+
+
+def clustered(c, n, seed=3):
+    """n particles: two thirds in a few cells, the others anywhere."""
+    rng = np.random.default_rng(seed)
+    p = {k: v[:n].copy() for k, v in c.oracle().particles().items()}
+    at = [rng.integers(0, c.N[q], n) for q in range(3)]
+    near = np.arange(n) % 3 > 0
+    for q in range(3):
+        at[q][near] = np.minimum(c.N[q] - 1, c.N[q] // 2 + at[q][near] % 3)
+    g, d = c.guard, c.dims
+    p["cell"] = ((at[0] + g[0]) + d[0] * ((at[1] + g[1]) + d[1] * (at[2] + g[2]))).astype(np.uint32)
+    return p
+
+
+@pytest.mark.parametrize("n", [300, 18000])
+@pytest.mark.parametrize("N", MESHES)
+def test_fp64_bit_exact(N, n):
+    c = Case(N, 1, theta=(0.1, 0.1), drift=(0.2, -0.2), Bbg=(0.3, 0.0, 1.0), data_interval=4)
+    p = clustered(c, n)
+    o = c.oracle(load=False)
+    o.set_particles(p)
+    env, d = c.gpu(precision=apt.APT_PREC_FP64, load=False)
+    d.set_particles(p)
+    o.sort()
+    d.sort_particles()
+    run_both(c, o, env, d, 6, sort_every=3)
+    assert_same_particles(d.get_particles(), o.particles())
+    assert_same_fields(d, o)
+
+
+@pytest.mark.parametrize("n", [300, 18000])
+@pytest.mark.parametrize("N", MESHES)
+def test_mixed_equals_unsorted_slots(N, n):
+    c = Case(N, 1, theta=(0.2, 0.2), drift=(0.3, -0.3), Bbg=(0.3, 0.0, 1.0), data_interval=3)
+    sims = []
+    for _ in range(2):
+        env = apt.sim_environment(apt.SimParams(
+            N=c.N, guard=c.guard, periodic_boundary=[False] * 3, max_ptc_number=n + 64,
+            precision=apt.APT_PREC_MIXED, data_interval=3))
+        sims.append((env, apt.sim_data(env)))
+    (env, a), (_, b) = sims
+    a.set_particles(clustered(c, n))
+    a.sort_particles()
+    b.set_particles(a.get_particles())
+    pu = apt.ptc_updater(env)
+    for step in range(3):
+        for d in (a, b):
+            pu.update_particles(d, c.dt, step)
+        for which in (apt.FIELD_J, apt.FIELD_RHO):
+            for comp in range(2):
+                assert np.array_equal(a.get_field(which, comp), b.get_field(which, comp)), step
