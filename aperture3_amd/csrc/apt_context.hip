@@ -366,7 +366,13 @@ static apt_status setup_tiles(apt_ctx *ctx) {
     ctx->tiles.nt[d] = 1;
     ctx->tiles.ax[d] = make_tile_axis(1, 1);
   }
-  for (int d = 0; d < 3; d++) ctx->tiles.T[d] = T[d];
+  ctx->tiles.shifts = true;
+  for (int d = 0; d < 3; d++) {
+    const TileAxis &a = ctx->tiles.ax[d];
+    ctx->tiles.T[d] = T[d];
+    ctx->tiles.sh[d] = a.dw.shift();
+    ctx->tiles.shifts = ctx->tiles.shifts && a.r == 0 && (a.w & (a.w - 1)) == 0;
+  }
   ctx->tiles.halo = halo;
   ctx->tiles.threads = threads;
   ctx->tiles.ntiles = (uint32_t)ntiles;

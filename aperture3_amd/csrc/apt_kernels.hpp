@@ -47,8 +47,6 @@ struct TileAxis {
   FastDiv dw, dw1;  // by w and by w + 1
   __host__ __device__ inline int origin(int t) const { return t * w + (t < r ? t : r); }
   __host__ __device__ inline int tile_of(int x) const {
-    // a shift for power-of-two extents without remainder (uniform branch)
-    if (r == 0 && (w & (w - 1)) == 0) return (int)((uint32_t)x >> dw.shift());
     const int s = r * (w + 1);
     return x < s ? (int)dw1.div((uint32_t)x) : r + (int)dw.div((uint32_t)(x - s));
   }
@@ -129,6 +127,11 @@ struct TileInfo {
   int T[3];       // largest tile extent in cells (the window is sized for it)
   int nt[3];      // tiles per dimension
   TileAxis ax[3];
+  // every axis in tiles of one power-of-two extent: tile = cell >> sh (3D, 16.7 M
+  // particles, us: count and scatter of a sort 83 + 475; 100 + 501 with a choice
+  // between shift and division made axis by axis)
+  bool shifts;
+  uint32_t sh[3];
   int halo;       // cells of LDS halo around a tile
   int threads;    // threads per tile workgroup
   const uint32_t *tile_off;

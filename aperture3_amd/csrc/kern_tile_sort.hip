@@ -41,9 +41,16 @@ __device__ __forceinline__ uint32_t tile_of_cell(const Mesh &m,
   int c1, c2, c3;
   m.split(c, c1, c2, c3);
   if (!m.in_bulk(c1, c2, c3)) return 0xffffffffu;
-  tc[0] = ti.ax[0].tile_of(c1 - m.guard[0]);
-  tc[1] = DIM > 1 ? ti.ax[1].tile_of(c2 - m.guard[1]) : 0;
-  tc[2] = DIM > 2 ? ti.ax[2].tile_of(c3 - m.guard[2]) : 0;
+  const uint32_t b[3] = {(uint32_t)(c1 - m.guard[0]), (uint32_t)(c2 - m.guard[1]),
+                         (uint32_t)(c3 - m.guard[2])};
+  // one uniform branch for all axes
+  if (ti.shifts) {
+#pragma unroll
+    for (int d = 0; d < 3; d++) tc[d] = d < DIM ? (int)(b[d] >> ti.sh[d]) : 0;
+  } else {
+#pragma unroll
+    for (int d = 0; d < 3; d++) tc[d] = d < DIM ? ti.ax[d].tile_of((int)b[d]) : 0;
+  }
   return (uint32_t)(tc[0] + ti.nt[0] * (tc[1] + ti.nt[1] * tc[2]));
 }
 
