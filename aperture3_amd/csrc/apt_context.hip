@@ -2443,12 +2443,16 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
     return APT_OK;
   }
   uint64_t kept = 0;
+  bool pay = true;
   if (by_runs) {  // the table's last entry, then the items and the slots in tiles
     uint32_t h[3];
     HIPCHK(hipMemcpyAsync(h, ctx->runs.work - 1, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     kept = h[0];
     ctx->runs.guard_slots = kept - h[2];
+    if (!ctx->logsph)
+      pay = ctx->prec == APT_PREC_FP64 ? f64_runs_pay(ctx->mesh.dim, kept, h[1])
+                                       : mixed_runs_pay(ctx->mesh.dim, kept, h[1]);
   } else {
     HIPCHK(hipMemcpyAsync(&kept, ctx->sortw.count, 8, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -2459,7 +2463,7 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
     HIPCHK(launch_fill<uint32_t>(cell + kept, MAX_CELL, n - kept, ctx->stream));
   }
   ctx->number = kept;
-  if (by_runs) {
+  if (by_runs && pay) {
     ctx->runs.end = kept;
     ctx->runs_valid = true;
   }

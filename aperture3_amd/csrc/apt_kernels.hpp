@@ -89,9 +89,12 @@ void cell_runs_shape(const Mesh &m, const int T[3], uint32_t least, CellRuns &cr
 hipError_t build_cell_runs(const Mesh &m, const CellRuns &cr, const uint32_t *keys, uint64_t n,
                            uint32_t *table, hipStream_t st);
 
-// tile extents of the updates over cell runs, by dimension
+// tile extents of the updates over cell runs, by dimension, and whether they are
+// the faster ones: kept slots in `items` work items
 void mixed_runs_tile(int dim, int T[3]);
+bool mixed_runs_pay(int dim, uint64_t kept, uint32_t items);
 void f64_runs_tile(int dim, int T[3]);
+bool f64_runs_pay(int dim, uint64_t kept, uint32_t items);
 // the update of the slots below cr.end, through LDS windows by tile
 hipError_t launch_push_deposit_f64_runs(const Mesh &m, const Species &sp, double dt, int H,
                                         int rho, const PtcF64 &p, const FieldsF64 &f,

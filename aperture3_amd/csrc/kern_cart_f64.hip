@@ -810,6 +810,16 @@ void f64_runs_tile(int dim, int T[3]) {
   T[2] = dim == 1 ? F64RunShape<1>::T2 : dim == 2 ? F64RunShape<2>::T2 : F64RunShape<3>::T2;
 }
 
+// As mixed_runs_pay, against the update of chunks of consecutive slots (us per
+// push, that one / this one): 1D, 62,500 tiles, 16 slots a tile 319 / 576, 32
+// 607 / 637, 64 1208 / 723; 2D, 65,536 tiles, 13 1398 / 2745, 64 3366 / 2977, but
+// 4096 tiles, 13 217 / 155 (the chunks then are too few to fill the chip); 3D,
+// 131,072 tiles, 6 2034 / 7001, 32 6164 / 7870, 16,384 tiles, 64 1654 / 1449.
+bool f64_runs_pay(int dim, uint64_t kept, uint32_t items) {
+  const uint64_t least = dim == 1 ? 40 : dim == 2 ? 48 : 64;
+  return items <= (dim == 2 ? 4096u : 1024u) || kept >= least * items;
+}
+
 // The FP64 update of cell-sorted slots: one workgroup per tile (or share of a
 // tile), the tile's current -- and, RHO, the charge of two species -- summed
 // in an LDS window over the tile and a halo that holds the drift of a sort

@@ -235,6 +235,17 @@ void mixed_runs_tile(int dim, int T[3]) {
   T[2] = dim == 3 ? 8 : 1;
 }
 
+// A workgroup clears and flushes a window whatever is in its tile, so on thin
+// plasma the update of one HBM atomic per contribution is the faster one, unless
+// there are so few tiles that either is a launch and little more.  The lines lie
+// where the two meet (us per push, that one / this one): 1D, 62,500 tiles, 8
+// slots a tile 105 / 229, 16 168 / 233, 32 333 / 237; 2D open, 4096 tiles, 13
+// 62 / 88, 128 223 / 109; 3D open, 1728 tiles, 26 78 / 188, 256 328 / 213.
+bool mixed_runs_pay(int dim, uint64_t kept, uint32_t items) {
+  const uint64_t least = dim == 1 ? 24 : dim == 2 ? 64 : 192;
+  return items <= (dim == 3 ? 256u : 1024u) || kept >= least * items;
+}
+
 // The mixed update of cell-sorted slots where the tiled push does not apply
 // (1D, and open axes): one workgroup per tile (or share of a tile), the current
 // and the charge of two species summed in an LDS window over the tile and a

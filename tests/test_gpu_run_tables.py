@@ -1,6 +1,6 @@
 """The tables of the updates over runs of sorted slots on meshes of many tiles:
 more than one workgroup of work items, tiles that hold most of the particles and
-are shared, tiles that are empty.  FP64 against the oracle bit for bit; mixed
+are shared, tiles that are empty, plasma too thin for them.  FP64 against the oracle bit for bit; mixed
 against a context that is given the sorted particles and never sorts."""
 import numpy as np
 import pytest
@@ -12,8 +12,9 @@ from test_gpu_parity_cart import assert_same_particles, run_both
 
 pytestmark = pytest.mark.gpu
 
-# 1D: 563 tiles of 16 cells; 2D: 325; 3D: 8 x 4 x 4 FP64, 8^3 mixed: 780, 120
-MESHES = [(9000,), (200, 390), (43, 41, 50)]
+# 1D: 563 tiles of 16 cells; 2D: 325; 3D: 8 x 4 x 4 FP64, 8^3 mixed: 780, 120.
+# 40,000 cells, 18,000 particles: thin on 2500 tiles, so not taken by tile
+MESHES = [(9000,), (200, 390), (43, 41, 50), (40000,)]
 
 
 def clustered(c, n, seed=3):
