@@ -72,6 +72,10 @@ struct apt_ctx {
   bool tiling = false;       // shape set up for this mesh
   bool tiles_valid = false;  // particles are binned by tile
   uint32_t pushes_since_sort = 0;  // eager tiled pushes since the binning
+  // 3D, shape not named by the caller: a small halo while the drift of light
+  // since the binning, in cells, is small (see setup_tiles)
+  bool tiles_by_drift = false;
+  double drift = 0.0;
   TileSortWork tsort;
 
   // runs of cell-sorted slots by tile (Cartesian FP64 and untiled mixed, 2D
@@ -315,17 +319,31 @@ static void free_ph32(PhoF32 &p) {
 // Shapes chosen here when the caller names none, from the mesh size.  The halo
 // has to hold the drift of a sort interval, since particles past it are
 // pushed one by one through HBM (16 x 16 + 6 against + 8: 12 M against 0.3 M
-// such pushes per 140 steps of 1024 x 768 cells at 32 per cell):
-//   2D, at least 512 tiles of 32 x 16: those, halo 8, 512 threads (1024 x 768:
-//   382 us per push, 16 x 16 + 6 with 256 threads 399; 1024^2 at 4 per cell
-//   92 against 129);
-//   2D below that: 16 x 16, halo 8 (128^2 at 32 per cell: 23 us against 26
-//   with 32 x 16 and 31 with halo 6);
-//   3D, at least 512 tiles of 8^3: halo 5, 1024 threads, one workgroup per CU
-//   (128^3 at 8 per cell 690 us, halo 4 with 512 threads 790, halo 3 with 256
-//   890);
-//   3D below that: halo 4, 512 threads (32 x 46 x 32 at 6 per cell: 29 us,
-//   halo 5 with 1024 threads 35).
+// such pushes per 140 steps of 1024 x 768 cells at 32 per cell).  Us per push,
+// one thing changed at a time (256 threads with halo 8 leave one workgroup's
+// worth of waves on a CU):
+//   2D, cells, per cell      16x16+6/256  16x16+8/256  16x16+8/512  32x16+8/512
+//       512 x 512,   8            50           83           43           49
+//       1024 x 256, 32           138          298          131          130
+//       1024 x 768,  2            63          106           57           56
+//       1024 x 768,  8           136          246          126          121
+//       1024 x 768, 32           405          881          395          395
+//       2048^2,     0.5          221          429          214          205
+//       2048^2,      4           461          862          390          371
+// so 16 x 16 + 8 with 512 threads below 1024 tiles of 32 x 16, those above it.
+// 3D, from 512 tiles of 8^3 on: halo 5, 1024 threads, one workgroup per CU; below
+// that halo 4, 512 threads (32 x 46 x 32 at 6 per cell: 29 us, halo 5 with 1024
+// threads 35).  The 3D window is large beside its tile, so while the halo of 3
+// holds the particles (up to a drift of 2.5 cells for light), and on thin plasma
+// always, the first of these is the faster one; us per push, sorted every 3, 5,
+// 10, 20 steps of half a cell:
+//   cells, per cell        8^3+3/256               8^3+5/1024
+//   128^3, 0.25      136  140  168  223       198  192  201  229
+//   128^3, 1         184  186  266  431       235  231  248  355
+//   128^3, 8         671  668  896 1845       693  685  739 1003
+//   256^3, 0.25     1081 1098 1356 1733      1548 1569 1660 1973
+//   256^3, 1        1476 1566 2032 3233      1949 2001 2160 2847
+//   256^3, 2        1919 2065 2742 4759      2386 2454 2671 4172
 static apt_status setup_tiles(apt_ctx *ctx) {
   const Mesh &m = ctx->mesh;
   const apt_params &pr = ctx->params;
@@ -336,7 +354,7 @@ static apt_status setup_tiles(apt_ctx *ctx) {
   const bool named = pr.tile[0] > 0 || pr.tile[1] > 0 || pr.tile_halo > 0 || pr.tile_threads > 0;
   auto tiles_of = [](int N, int t) { return (uint64_t)((N + t - 1) / t); };
   if (m.dim == 2) {
-    const bool wide = !named && tiles_of(m.N[0], 32) * tiles_of(m.N[1], 16) >= 512;
+    const bool wide = !named && tiles_of(m.N[0], 32) * tiles_of(m.N[1], 16) >= 1024;
     T[0] = pr.tile[0] > 0 ? pr.tile[0] : (wide ? 32 : 16);
     T[1] = pr.tile[1] > 0 ? pr.tile[1] : 16;
     halo = T[0] == 8 ? 4 : 6;
@@ -351,6 +369,7 @@ static apt_status setup_tiles(apt_ctx *ctx) {
       const bool many = tiles_of(m.N[0], 8) * tiles_of(m.N[1], 8) * tiles_of(m.N[2], 8) >= 512;
       halo = many ? 5 : 4;
       threads = many ? 1024 : 512;
+      ctx->tiles_by_drift = many;
     }
   }
   if (ctx->params.tile_halo > 0) halo = ctx->params.tile_halo;
@@ -1232,6 +1251,7 @@ apt_status apt_ptc_load_uniform(apt_ctx *ctx, int ppc_pairs,
     HIPCHK(hipMemcpyAsync(ctx->tile_off, off.data(), off.size() * 4,
                           hipMemcpyHostToDevice, ctx->stream));
     ctx->tiles.tiled_end = add;
+    ctx->drift = 0.0;
     ctx->tiles_valid = true;
     ctx->pushes_since_sort = 0;
   }
@@ -1811,6 +1831,16 @@ apt_status apt_ptc_update(apt_ctx *ctx, double dt, uint32_t step) {
       ctx->pushes_since_sort++;
     }
     TileInfo ti = ctx->tiles;
+    if (ctx->tiles_by_drift) {
+      // a recorded step takes the large halo: it may be replayed at any drift
+      double step_cells = 0.0;
+      for (int d = 0; d < 3; d++) step_cells = fmax(step_cells, fabs(dt) * ctx->mesh.inv_delta[d]);
+      if (!ctx->capturing) ctx->drift += step_cells;
+      if ((!ctx->capturing && ctx->drift <= 2.5) || ti.tiled_end < 192ull * ti.ntiles) {
+        ti.halo = 3;
+        ti.threads = 256;
+      }
+    }
     if (!ctx->tiles_valid) {
       ti.tile_off = nullptr;
       ti.ntiles = 0;
@@ -2306,6 +2336,7 @@ static apt_status sort_tiles(apt_ctx *ctx) {
   ti.tiled_end = kept;
   ctx->tiles_valid = true;
   ctx->pushes_since_sort = 0;
+  ctx->drift = 0.0;
   return APT_OK;
 }
 
@@ -2872,6 +2903,7 @@ apt_status apt_graph_launch(apt_ctx *ctx, int times) {
   if (!ctx->gexec) return ctx->fail(APT_ERR_STATE, "graph_launch: no recorded step");
   if (ctx->capturing) return ctx->fail(APT_ERR_STATE, "graph_launch: a step is recorded");
   ctx->rho_zero = false;  // a recorded deposit step writes Rho
+  ctx->drift = 1e30;      // and moves the particles on
   for (int k = 0; k < times; k++) HIPCHK(hipGraphLaunch(ctx->gexec, ctx->stream));
   return APT_OK;
 }
