@@ -1277,11 +1277,21 @@ static hipError_t launch_logsph_push(const Mesh &m, const Species &sp, const LsP
   if (n == 0) return hipSuccess;
   const uint32_t nwork = runs ? runs->items : 0;
   const uint64_t rest = runs && !dn ? n - runs->end : n;
-  uint64_t tail = (rest + LS_NT - 1) / LS_NT;
-  // under a bound nearly all of these are past the count, and each holds 40 KB
-  // of LDS while it finds out: 1024 x 1024 with
-  // pairs, 0.42 -> 0.32 ms a push
-  if (dn && tail > LS_DEV_TAIL) tail = LS_DEV_TAIL;
+  // Slots of a workgroup behind the tiles, a slot a thread if they can be: the
+  // cells of many do not fit the window.  Before a sort every slot is there, and
+  // from 16 to a cell on two a thread cover no more cells (us per push, slots in
+  // cell order, FP32, 1024 x 1024: 4 M 468 with 512, 577 with 1024; 24 M 2355,
+  // 2086; 512 x 512: 8 M 820, 762).
+  // Under a bound nearly all of the workgroups behind sorted slots are past the
+  // count, and each holds 40 KB of LDS while it finds out: there are at most 4096
+  // (1024 x 1024 with pairs, 0.42 -> 0.32 ms a push) or one for 4096 slots of the
+  // bound, and a thread takes several slots where the count needs it.
+  uint64_t slots = runs == nullptr && rest >= 16 * m.size() ? 2 * LS_NT : LS_NT;
+  if (dn && runs) {
+    slots = (rest + LS_DEV_TAIL - 1) / LS_DEV_TAIL;
+    slots = slots < LS_NT ? LS_NT : slots > 4096 ? 4096 : slots;
+  }
+  uint64_t tail = (rest + slots - 1) / slots;
   if (tail == 0) tail = 1;  // the guard rows above the tiles
   const uint64_t grid = nwork + (runs ? 1 : 0) + tail;
   const CellRuns cr = runs ? *runs : CellRuns{};
