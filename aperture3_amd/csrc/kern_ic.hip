@@ -895,10 +895,13 @@ static apt_status ic_sample_dev(apt_ic *h, const double *gamma, double *eph, uin
   if (n > IC_MAX_SAMPLES) return h->fail(APT_ERR_INVALID_ARG, "ic sampling: too many samples");
   hipStream_t st = stream ? (hipStream_t)stream : h->stream;
   const uint64_t blocks = (n + 255) / 256;
-  if (h->d_guide) {
-    // a workgroup copies the small tables to LDS, so past 8 per CU it takes
-    // several rounds of samples
-    const size_t lds = (size_t)h->ng * 16 + (size_t)(h->nep + 1) * sizeof(IcPath);
+  // A workgroup copies the small tables to LDS, so past 8 per CU it takes several
+  // rounds of samples.  With large tables and a round each the copy costs more
+  // than the guide saves (us, plain / guided: 2048 x 2048, 32,768 samples 11.1 /
+  // 12.1, 262,144 21.2 / 25.2, 524,288 39.7 / 38.8; 1200 x 1200, 32,768 10.0 /
+  // 10.6, 262,144 18.3 / 14.9).
+  const size_t lds = (size_t)h->ng * 16 + (size_t)(h->nep + 1) * sizeof(IcPath);
+  if (h->d_guide && (lds <= 32768 || blocks >= 2048)) {
     k_ic_sample_guided<<<(unsigned)(blocks < 2048 ? blocks : 2048), 256, lds, st>>>(
         tables_of(h), gamma, eph, n, seed, epoch, accept);
   } else {
