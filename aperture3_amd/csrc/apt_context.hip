@@ -698,6 +698,7 @@ apt_status apt_create(const apt_grid *grid, const apt_params *params,
     apt_destroy(ctx);
     return APT_ERR_INVALID_ARG;
   }
+  ctx->sortw.most = ctx->rtw.most = ctx->cap > ctx->ph_cap ? ctx->cap : ctx->ph_cap;
   if (ctx->ph_cap > 0 && (st = alloc_photons(ctx, false)) != APT_OK) {
     apt_destroy(ctx);
     return st;
@@ -2348,6 +2349,15 @@ static apt_status sort_photons(apt_ctx *ctx) {
   if (ctx->capturing) return ctx->fail(APT_ERR_STATE, "sort: not while a step is recorded");
   if (!ctx->ph_have_b) {
     apt_status st = alloc_photons(ctx, true);
+    if (st != APT_OK) {
+      // the particles' sort before may have left more room than this one needs
+      (void)hipGetLastError();
+      free_ph64(ctx->ph64b);
+      free_ph32(ctx->ph32b);
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+      ctx->sortw.release();
+      st = alloc_photons(ctx, true);
+    }
     if (st != APT_OK) return st;
     ctx->ph_have_b = true;
   }

@@ -383,6 +383,7 @@ struct RtWork {
   unsigned long long *total = nullptr, *host_total = nullptr;  // the latter pinned
   uint64_t *bsum = nullptr;  // per-workgroup event prefixes
   uint64_t cap = 0;
+  uint64_t most = 0;  // slots its owner can ever have: no room beyond
   hipError_t ensure(uint64_t n);
   hipError_t alloc(uint64_t c);
   void release();

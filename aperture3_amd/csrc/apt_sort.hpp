@@ -4,6 +4,14 @@
 
 namespace apt {
 
+// Slots to have room for when n are needed now: half as much again for a count
+// that grows, but no more than there can ever be (a set that fills its capacity
+// takes what it needs and no more).
+inline uint64_t room_for(uint64_t n, uint64_t most) {
+  const uint64_t s = n + n / 2;
+  return s < most ? s : n > most ? n : most;
+}
+
 struct SortWork {
   uint32_t *keys_in = nullptr, *keys_out = nullptr;
   uint32_t *perm_in = nullptr, *perm_out = nullptr;
@@ -11,6 +19,7 @@ struct SortWork {
   void *temp = nullptr;
   size_t temp_bytes = 0;
   uint64_t cap = 0;
+  uint64_t most = 0;  // slots its owner can ever have: no room beyond
   hipError_t ensure(uint64_t n);
   hipError_t alloc(uint64_t n);
   void release();
@@ -29,7 +38,6 @@ hipError_t sort_keys(SortWork &w, const uint32_t *cell, uint64_t n,
 hipError_t hipcub_sort_pairs(SortWork &w, uint64_t n, int bits,
                              hipStream_t st);
 
-// dst[i] = src[perm_out[i]]
 // The arrays of a particle set, gathered into sorted order together.
 struct GatherSet {
   static constexpr int MAX4 = 12, MAX8 = 12;

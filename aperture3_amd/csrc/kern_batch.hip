@@ -1271,6 +1271,7 @@ static apt_status batch_sort(apt_batch *b, int photons) {
   const uint64_t total = photons ? b->ph_cap : b->cap;
   if (total == 0) return APT_OK;
   SortWork &w = b->sortw;
+  w.most = b->cap > b->ph_cap ? b->cap : b->ph_cap;
   BCHK(w.ensure(total));
   const uint32_t *cell = photons ? (b->prec == APT_PREC_FP64 ? b->h64.cell : b->h32.cell)
                                  : (b->prec == APT_PREC_FP64 ? b->p64.cell : b->p32.cell);

@@ -18,6 +18,7 @@
 
 #include "apt_common.hpp"
 #include "apt_kernels.hpp"
+#include "apt_sort.hpp"
 #include "apt_math.hpp"
 
 namespace apt {
@@ -511,13 +512,15 @@ static inline unsigned rt_blocks(uint64_t n) {
 }
 
 // A run's counts grow with every injection: sized to the count, the scratch was
-// freed and allocated again on each call, ~100 us a step.  Half as much again,
-// or just n where memory is short.
+// freed and allocated again on each call, ~100 us a step.  So room_for(n), or just
+// n where memory is short.
 hipError_t RtWork::ensure(uint64_t n) {
   if (n <= cap && host_total) return hipSuccess;
-  const uint64_t least = n < 1024 ? 1024 : n;
-  if (alloc(least + least / 2) == hipSuccess) return hipSuccess;
-  (void)hipGetLastError();
+  const uint64_t least = n < 1024 ? 1024 : n, slack = room_for(least, most);
+  if (slack > least) {
+    if (alloc(slack) == hipSuccess) return hipSuccess;
+    (void)hipGetLastError();
+  }
   return alloc(least);
 }
 

@@ -172,9 +172,11 @@ int key_bits(uint32_t max_key) {
 // room for a growing count, as RtWork::ensure
 hipError_t SortWork::ensure(uint64_t n) {
   if (n <= cap) return hipSuccess;
-  const uint64_t slack = n + n / 2;
-  if (slack <= 0x7fffffffull && alloc(slack) == hipSuccess) return hipSuccess;
-  (void)hipGetLastError();
+  const uint64_t slack = room_for(n, most);
+  if (slack > n && slack <= 0x7fffffffull) {
+    if (alloc(slack) == hipSuccess) return hipSuccess;
+    (void)hipGetLastError();
+  }
   return alloc(n);
 }
 
