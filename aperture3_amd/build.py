@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import concurrent.futures as cf
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -59,12 +60,36 @@ HIPCC_FLAGS = [
 ]
 
 
+RESOURCE_REMARKS = ["-Rpass-analysis=kernel-resource-usage"]
+
+
 def _hipcc() -> str:
     for cand in (os.environ.get("HIPCC"), shutil.which("hipcc"),
                  "/opt/rocm/bin/hipcc"):
         if cand and os.path.exists(cand):
             return cand
     raise RuntimeError("hipcc not found: the HIP library cannot be built")
+
+
+# Kernels compiled for a stated number of waves per SIMD.  A build of the FP64
+# log-spherical push that spilled vector registers to stay within its number
+# gave wrong particles, so a compiler that would spill here is refused.
+NO_SPILL = ("k_logsph_push", "k_push_deposit_f64_runs", "k_push_deposit_f64_win")
+
+
+def spilling_kernels(remarks: str) -> list[str]:
+    """The NO_SPILL kernels that the compiler's kernel-resource-usage remarks
+    report vector register spills for."""
+    bad, name = [], ""
+    for line in remarks.splitlines():
+        m = re.search(r"remark: .*?(Function Name|VGPRs Spill): (\S+)", line)
+        if not m:
+            continue
+        if m[1] == "Function Name":
+            name = m[2]
+        elif m[2] != "0" and any(k in name for k in NO_SPILL):
+            bad.append(f"{name}: {m[2]} spills")
+    return bad
 
 
 def _run(cmd: list[str]) -> None:
@@ -74,6 +99,10 @@ def _run(cmd: list[str]) -> None:
                     if "packed-fp32-ops" not in l and "not a recognized feature" not in l)
     if res.returncode != 0:
         raise RuntimeError(f"build failed: {' '.join(cmd)}\n{out}")
+    spills = spilling_kernels(res.stdout)
+    if spills:
+        raise RuntimeError("build refused, vector registers spilled in kernels compiled "
+                           "for a stated occupancy:\n" + "\n".join(spills))
 
 
 # The mixed-precision kernels use the hardware FP32 reciprocal/square root
@@ -93,7 +122,8 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
     for src in HIP_SOURCES + HOST_SOURCES:
         obj = os.path.join(BUILD, src.replace("/", "_") + ".o")
         objs.append(obj)
-        cmds.append([hipcc, *HIPCC_FLAGS, *FILE_FLAGS.get(src, []), "-c",
+        cmds.append([hipcc, *HIPCC_FLAGS, *FILE_FLAGS.get(src, []),
+                     *(RESOURCE_REMARKS if src.endswith(".hip") else []), "-c",
                      os.path.join(CSRC, src), "-o", obj])
     jobs = jobs or min(8, os.cpu_count() or 4)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:

@@ -494,7 +494,10 @@ constexpr int ls_win() {
 
 // waves per SIMD asked of the compiler: two workgroups per CU (FP64: 126 VGPRs;
 // with the 130 it takes unasked, one workgroup and 188 us for 131), except on
-// FP64 charge steps, which do not fit in 128 VGPRs without spilling
+// FP64 charge steps, which do not fit in 128 VGPRs without spilling: compiled so,
+// they gave wrong particles in all waves of a workgroup but the first, for a
+// reason that was not found (the spill and its reloads read right), so that form
+// is not built and the build refuses spills here (build.py)
 template <typename R, bool RHO>
 constexpr int ls_waves() {
   return std::is_same<R, double>::value && RHO ? 2 : 4;
