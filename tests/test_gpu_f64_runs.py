@@ -1,7 +1,7 @@
 """GPU tests of the FP64 update over runs of cell-sorted slots (LDS windows by
 tile): bit-exact against the oracle on meshes that are no multiples of the
 tile, smaller than a tile or than its window, open and periodic, with charge
-output, slots appended after the sort, particles in guard cells, and fields
+output, a load after the sort, particles in guard cells, and fields
 that are not finite."""
 import ctypes as C
 
@@ -109,7 +109,8 @@ def test_runs_with_fields_that_are_not_finite(N, value):
 
 def test_runs_with_guard_cells_and_an_unsorted_tail():
     """Particles in guard cells are sorted with the others and erased by the
-    next push; a second load after the sort is pushed from its own slots."""
+    next push; a second load after a sort leaves every slot to the update of
+    consecutive slots (slots behind sorted ones: test_gpu_run_tails)."""
     for N in ((20,), (18, 10), (8, 7, 6)):
         c = Case(N, 2, theta=(0.1, 0.1), drift=(0.2, -0.2), Bbg=(0.3, 0.0, 1.0))
         o = c.oracle()
@@ -127,7 +128,7 @@ def test_runs_with_guard_cells_and_an_unsorted_tail():
         assert np.array_equal(pg["cell"], ps["cell"])
         assert (ps["cell"] == apt.MAX_CELL).sum() == len(guard)
         assert_same_fields(d, o, rho=False)
-        # the tail: slots appended past the sorted ones, pushed with them
+        # a second load: no slot is taken by tile any more
         before = d.get_particles()
         live = before["cell"] != apt.MAX_CELL
         d.sort_particles()

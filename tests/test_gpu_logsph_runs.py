@@ -69,8 +69,9 @@ def test_mixed_sorted_equals_unsorted(kind, N, nptc):
 
 
 def test_device_counts_more_slots_than_the_grid():
-    """Under a device count the workgroups behind the tiles are capped, and each
-    takes several slots a thread: the same integer sums as with host counts."""
+    """Slots never sorted, 512 to a cell, two a thread: the same integer sums
+    under a device count as with host counts (behind sorted slots, where a device
+    count caps the workgroups: test_gpu_run_tails)."""
     c = LogSphCase(N=(64, 64), nptc=4096 * 512 + 70001, damping_length=6)
     out = []
     for device in (False, True):

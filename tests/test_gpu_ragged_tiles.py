@@ -82,7 +82,7 @@ def test_ragged_step_vs_oracle(N, ppc, tile, halo, threads):
     assert np.array_equal(tg, ts)
     same = pg["cell"] == ps["cell"]
     assert np.mean(same) > 0.999
-    for k in ("x1", "x2"):
+    for k in ("x1", "x2", "x3")[:max(2, len(N))]:
         assert np.abs(pg[k][same] - ps[k][same]).max() < 1e-4, k
     for k in ("p1", "p2", "p3"):
         assert np.abs(pg[k] - ps[k]).max() <= 1e-5 * np.abs(ps[k]).max(), k
