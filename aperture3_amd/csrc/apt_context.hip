@@ -870,14 +870,14 @@ static void **field_slot(apt_ctx *ctx, int which, int comp) {
   return nullptr;
 }
 
-// the Cartesian force-free work fields, zeroed, on first use
-// a field other than through a step's own kernels
+// a field was written other than through a step's own kernels
 static void field_written(apt_ctx *ctx, int which) {
   if (which == APT_FIELD_EBG) ctx->ebg_zero = false;
   if (which == APT_FIELD_BBG) ctx->bbg_zero = false;
   if (which == APT_FIELD_RHO) ctx->rho_zero = false;
 }
 
+// the Cartesian force-free work fields, zeroed, on first use
 static hipError_t ensure_ffe_cart(apt_ctx *ctx, int n = 7) {
   const size_t es = ctx->prec == APT_PREC_FP64 ? 8 : 4;
   for (int k = 0; k < n; k++) {

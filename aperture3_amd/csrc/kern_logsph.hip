@@ -971,8 +971,9 @@ __device__ inline void axis_upper(const Mesh &m, const FieldSet<T> &f, int i) {
   B1[b] = (B1[a] - H1[a]) + H1[b];
 }
 
-// The boundary rules in one launch (512 x 512: 16 us in four, 9.6 in one).  A column's axis rows go through every rule, in order, in one
-// thread; the star's and the outflow layer's other cells have a thread each.
+// The boundary rules in one launch (512 x 512: 16 us in four, 9.6 in one).  A
+// column's axis rows go through every rule, in order, in one thread; the star's
+// and the outflow layer's other cells have a thread each.
 template <typename T>
 __global__ void k_logsph_boundary(Mesh m, LsParams lp, FieldSet<T> f, double omega) {
   const int d0 = m.dims[0], d1 = m.dims[1], g0 = m.guard[0], L = lp.damping_length;
