@@ -46,8 +46,10 @@ __global__ void k_count_valid(const uint32_t *__restrict__ keys, uint64_t n,
 // All arrays of a particle set in one pass: the permutation is read once, and a
 // slot's loads, which depend on nothing but it, are in flight together.  With a
 // launch per array the loads of one array waited for the last one's grid to
-// drain: eight 1D boxes, 7 M slots, 45 launches of 65-70 us; a pass of 20 steps
-// with one sort 11.4 -> 11.0 ms.
+// drain: eight 1D boxes, 26 M particles and their photons, 19 launches of 62-67 us
+// on average, 1.2 ms a sort; 0.75 ms in two; a pass of 20 steps with one sort 11.4
+// -> 10.9 ms.  638 M particles take as long as before (9 x 1.5 ms), as do 17 M in
+// random order (9 x 295 us): the gathered lines are the bound there.
 template <int N4, int N8>
 __global__ void k_gather_set(GatherSet g, const uint32_t *__restrict__ perm, uint64_t n) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
