@@ -2428,8 +2428,10 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
   if (st != APT_OK) return st;
   const uint32_t empty_key = (uint32_t)ctx->ncell;
   if (ctx->prec == APT_PREC_MIXED && ctx->tiling) return sort_tiles(ctx);
-  // the updates that walk runs of sorted slots (the log-spherical one is 2D)
-  const bool by_runs = ctx->logsph ? ctx->mesh.dim == 2 : !ctx->gr1d && !ctx->gap1d;
+  // the updates that walk runs of sorted slots (the log-spherical one is 2D, in
+  // the mesh's first plane)
+  const bool by_runs = ctx->logsph ? ctx->mesh.dim == 2 && ctx->mesh.dims[2] == 1
+                                   : !ctx->gr1d && !ctx->gap1d;
   time_begin(ctx, APT_KERNEL_SORT);
   if (ctx->prec == APT_PREC_FP64) {
     PtcF64 &a = ctx->p64, &b = ctx->p64b;
@@ -2491,7 +2493,9 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
     HIPCHK(hipStreamSynchronize(ctx->stream));
     kept = h[0];
     ctx->runs.guard_slots = kept - h[2];
-    if (!ctx->logsph)
+    if (ctx->mesh.dim == 1 && ctx->runs.guard_slots > 0)
+      pay = false;  // rows beside a 1D mesh: no kernel of their own
+    else if (!ctx->logsph)
       pay = ctx->prec == APT_PREC_FP64 ? f64_runs_pay(ctx->mesh.dim, kept, h[1])
                                        : mixed_runs_pay(ctx->mesh.dim, kept, h[1]);
   } else {

@@ -7,6 +7,7 @@ import pytest
 
 import aperture3_amd as apt
 from cases import Case
+from logsph_cases import LogSphCase
 from test_gpu_f64_runs import assert_same_fields
 from test_gpu_parity_cart import assert_same_particles, run_both
 
@@ -67,3 +68,33 @@ def test_mixed_equals_unsorted_slots(N, n):
         for which in (apt.FIELD_J, apt.FIELD_RHO):
             for comp in range(2):
                 assert np.array_equal(a.get_field(which, comp), b.get_field(which, comp)), step
+
+
+@pytest.mark.parametrize("precision", [apt.APT_PREC_FP64, apt.APT_PREC_MIXED])
+def test_log_spherical_mesh_with_guard_planes(precision):
+    """Guard cells along the axis that a 2D mesh does not have: the step lives in
+    the first plane, sorted or not."""
+    c = LogSphCase(N=(40, 33), nptc=4000, damping_length=6, data_interval=1)
+    out = []
+    for planes in (0, 1):
+        env = apt.sim_environment(apt.SimParams(
+            N=[40, 33, 1], guard=c.guard[:2] + [planes], size=c.size, num_species=3,
+            max_ptc_number=c.cap, precision=precision, data_interval=1,
+            coord_system="LogSpherical", omega=0.1, B0=c.mu, damping_length=6))
+        d = apt.sim_data(env)
+        n = c.ncell
+        for q, f in enumerate(c.dipole()):
+            full = np.zeros(env.ncell())
+            full[:n] = f
+            d.set_field(apt.FIELD_BBG, q, full)
+            d.set_field(apt.FIELD_B, q, full)
+        d.set_particles(c.particles())
+        d.sort_particles()
+        pu = apt.ptc_updater_logsph(env)
+        for step in range(2):
+            pu.update_particles(d, c.dt, step)
+        out.append([d.get_field(apt.FIELD_J, q)[:n] for q in range(3)] +
+                   [d.get_particles()["x1"]])
+    assert np.abs(out[0][0]).max() > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b, equal_nan=True)
