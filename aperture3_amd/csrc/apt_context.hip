@@ -265,6 +265,24 @@ static apt_status alloc_ptc(apt_ctx *ctx, bool second) {
   return APT_OK;
 }
 
+static void drop_ftmp(apt_ctx *ctx) {
+  for (void *&q : ctx->ftmp) {
+    (void)hipFree(q);
+    q = nullptr;
+  }
+  (void)hipGetLastError();  // of the allocation that did not fit
+}
+
+// Memory that the context can do without, given back for an allocation that did
+// not fit: the sort's scratch, which may hold more room than is needed, and the
+// smoothing's work arrays, unless a recorded step holds them.
+static apt_status give_back(apt_ctx *ctx) {
+  HIPCHK(hipStreamSynchronize(ctx->stream));
+  ctx->sortw.release();
+  if (!ctx->gexec && !ctx->capturing) drop_ftmp(ctx);
+  return APT_OK;
+}
+
 static void free_ptc64(PtcF64 &p) {
   (void)hipFree(p.cell); (void)hipFree(p.x1); (void)hipFree(p.x2); (void)hipFree(p.x3);
   (void)hipFree(p.p1); (void)hipFree(p.p2); (void)hipFree(p.p3); (void)hipFree(p.E); (void)hipFree(p.w);
@@ -569,8 +587,6 @@ apt_status apt_create(const apt_grid *grid, const apt_params *params,
   ok = ok && alloc_field(&ctx->divE) && alloc_field(&ctx->divB) &&
        alloc_field(&ctx->jtmp) && alloc_field(&ctx->EdotB) &&
        alloc_field(&ctx->ph_produced) && alloc_field(&ctx->pair_produced);
-  if (params->coord == APT_COORD_CARTESIAN && params->current_smoothing > 0 && guard_images_ok(m))
-    for (int q = 0; q < 3 && ok; q++) ok = alloc_field(&ctx->ftmp[q]);
   int limbs = ctx->prec == APT_PREC_FP64 ? 2 : 1;
   for (int c = 0; c < 3 && ok; c++)
     for (int l = 0; l < limbs && ok; l++)
@@ -709,6 +725,14 @@ apt_status apt_create(const apt_grid *grid, const apt_params *params,
       apt_destroy(ctx);
       return st;
     }
+  }
+  // a smoothed box's work arrays last: where they do not fit, each component is
+  // filtered through jtmp in turn
+  if (params->coord == APT_COORD_CARTESIAN && params->current_smoothing > 0 &&
+      guard_images_ok(m)) {
+    bool room = true;
+    for (int q = 0; q < 3 && room; q++) room = alloc_field(&ctx->ftmp[q]);
+    if (!room) drop_ftmp(ctx);
   }
   if (hipStreamSynchronize(ctx->stream) != hipSuccess) {
     apt_destroy(ctx);
@@ -1315,7 +1339,7 @@ static apt_status smooth(apt_ctx *ctx, int rho) {
 template <typename T>
 static apt_status finalize_smooth(apt_ctx *ctx, int rho) {
   const int passes = ctx->params.current_smoothing, ns = ctx->params.num_species;
-  const bool fused = passes > 0 && guard_images_ok(ctx->mesh);
+  const bool fused = passes > 0 && ctx->ftmp[2] && guard_images_ok(ctx->mesh);
   T *tmp[4] = {(T *)ctx->jtmp, (T *)ctx->ftmp[0], (T *)ctx->ftmp[1], (T *)ctx->ftmp[2]};
   const bool odd = fused && (passes & 1);
   auto run = [&](void *const *field, int n) -> apt_status {
@@ -2233,6 +2257,12 @@ apt_status apt_field_compute_divs(apt_ctx *ctx) {
 static apt_status ensure_second_buffer(apt_ctx *ctx) {
   if (ctx->have_b) return APT_OK;
   apt_status st = alloc_ptc(ctx, true);
+  if (st != APT_OK) {
+    free_ptc64(ctx->p64b);
+    free_ptc32(ctx->p32b);
+    st = give_back(ctx);
+    if (st == APT_OK) st = alloc_ptc(ctx, true);
+  }
   if (st != APT_OK) return st;
   ctx->have_b = true;
   return APT_OK;
@@ -2350,13 +2380,10 @@ static apt_status sort_photons(apt_ctx *ctx) {
   if (!ctx->ph_have_b) {
     apt_status st = alloc_photons(ctx, true);
     if (st != APT_OK) {
-      // the particles' sort before may have left more room than this one needs
-      (void)hipGetLastError();
       free_ph64(ctx->ph64b);
       free_ph32(ctx->ph32b);
-      HIPCHK(hipStreamSynchronize(ctx->stream));
-      ctx->sortw.release();
-      st = alloc_photons(ctx, true);
+      st = give_back(ctx);
+      if (st == APT_OK) st = alloc_photons(ctx, true);
     }
     if (st != APT_OK) return st;
     ctx->ph_have_b = true;
@@ -2420,6 +2447,29 @@ apt_status apt_sort_particles(apt_ctx *ctx) {
   return sort_photons(ctx);
 }
 
+// The run table, at the first sort; false where it does not fit: the updates then
+// take consecutive slots.
+static bool make_run_table(apt_ctx *ctx) {
+  int T[3];
+  if (ctx->prec == APT_PREC_FP64)
+    f64_runs_tile(ctx->mesh.dim, T);
+  else
+    mixed_runs_tile(ctx->mesh.dim, T);
+  // a log-spherical tile is shared later: its particles cluster, and each share
+  // flushes a window (a cloud on half of the tiles: 78 us a push with 512, 70 with
+  // 2048; FP64 152, 140)
+  cell_runs_shape(ctx->mesh, T, ctx->logsph ? 2048 : 512, ctx->runs);
+  const uint64_t entries = cell_runs_size(ctx->mesh, ctx->runs);
+  if (hipMalloc(&ctx->run_off, (entries + 2 + 2 * (uint64_t)ctx->runs.items) * 4) != hipSuccess) {
+    (void)hipGetLastError();
+    ctx->run_off = nullptr;
+    return false;
+  }
+  ctx->runs.off = ctx->run_off;
+  ctx->runs.work = ctx->run_off + entries;
+  return true;
+}
+
 static apt_status sort_particles_only(apt_ctx *ctx) {
   uint64_t n = ctx->number;
   if (n == 0) return APT_OK;
@@ -2430,8 +2480,9 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
   if (ctx->prec == APT_PREC_MIXED && ctx->tiling) return sort_tiles(ctx);
   // the updates that walk runs of sorted slots (the log-spherical one is 2D, in
   // the mesh's first plane)
-  const bool by_runs = ctx->logsph ? ctx->mesh.dim == 2 && ctx->mesh.dims[2] == 1
-                                   : !ctx->gr1d && !ctx->gap1d;
+  bool by_runs = ctx->logsph ? ctx->mesh.dim == 2 && ctx->mesh.dims[2] == 1
+                             : !ctx->gr1d && !ctx->gap1d;
+  if (by_runs && !ctx->run_off) by_runs = make_run_table(ctx);
   time_begin(ctx, APT_KERNEL_SORT);
   if (ctx->prec == APT_PREC_FP64) {
     PtcF64 &a = ctx->p64, &b = ctx->p64b;
@@ -2452,21 +2503,6 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
   }
   ctx->runs_valid = false;
   if (by_runs) {
-    if (!ctx->run_off) {
-      int T[3];
-      if (ctx->prec == APT_PREC_FP64)
-        f64_runs_tile(ctx->mesh.dim, T);
-      else
-        mixed_runs_tile(ctx->mesh.dim, T);
-      // a log-spherical tile is shared later: its particles cluster, and each
-      // share flushes a window (a cloud on half of the tiles: 78 us a push with
-      // 512, 70 with 2048; FP64 152, 140)
-      cell_runs_shape(ctx->mesh, T, ctx->logsph ? 2048 : 512, ctx->runs);
-      const uint64_t entries = cell_runs_size(ctx->mesh, ctx->runs);
-      HIPCHK(hipMalloc(&ctx->run_off, (entries + 2 + 2 * (uint64_t)ctx->runs.items) * 4));
-      ctx->runs.off = ctx->run_off;
-      ctx->runs.work = ctx->run_off + entries;
-    }
     HIPCHK(build_cell_runs(ctx->mesh, ctx->runs, ctx->sortw.keys_out, n, ctx->run_off,
                            ctx->stream));
   }
