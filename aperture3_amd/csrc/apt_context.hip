@@ -328,6 +328,14 @@ static void free_ph32(PhoF32 &p) {
   p = PhoF32{};
 }
 
+// no guard cells along an axis that the mesh does not have (the updates of such a
+// mesh differ in the rows and planes beside it that they read)
+static bool no_idle_guards(const Mesh &m) {
+  for (int d = m.dim; d < 3; d++)
+    if (m.dims[d] != 1) return false;
+  return true;
+}
+
 // Tiling of the mixed form: every tiled dimension periodic; an axis whose N
 // is not a multiple of the tile extent is split evenly over ceil(N / extent)
 // tiles.  (Before, such a mesh took the untiled push with one HBM atomic per
@@ -395,6 +403,7 @@ static apt_status setup_tiles(apt_ctx *ctx) {
   uint64_t ntiles = 1;
   for (int d = 0; d < m.dim; d++) {
     if (!m.periodic[d]) return APT_OK;
+    if (m.N[d] % T[d] != 0 && !no_idle_guards(m)) return APT_OK;
     ctx->tiles.nt[d] = (m.N[d] + T[d] - 1) / T[d];
     ctx->tiles.ax[d] = make_tile_axis(m.N[d], ctx->tiles.nt[d]);
     ntiles *= (uint64_t)ctx->tiles.nt[d];
@@ -2478,10 +2487,9 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
   if (st != APT_OK) return st;
   const uint32_t empty_key = (uint32_t)ctx->ncell;
   if (ctx->prec == APT_PREC_MIXED && ctx->tiling) return sort_tiles(ctx);
-  // the updates that walk runs of sorted slots (the log-spherical one is 2D, in
-  // the mesh's first plane)
-  bool by_runs = ctx->logsph ? ctx->mesh.dim == 2 && ctx->mesh.dims[2] == 1
-                             : !ctx->gr1d && !ctx->gap1d;
+  // the updates that walk runs of sorted slots (the log-spherical one is 2D)
+  bool by_runs = no_idle_guards(ctx->mesh) &&
+                 (ctx->logsph ? ctx->mesh.dim == 2 : !ctx->gr1d && !ctx->gap1d);
   if (by_runs && !ctx->run_off) by_runs = make_run_table(ctx);
   time_begin(ctx, APT_KERNEL_SORT);
   if (ctx->prec == APT_PREC_FP64) {
@@ -2529,9 +2537,7 @@ static apt_status sort_particles_only(apt_ctx *ctx) {
     HIPCHK(hipStreamSynchronize(ctx->stream));
     kept = h[0];
     ctx->runs.guard_slots = kept - h[2];
-    if (ctx->mesh.dim == 1 && ctx->runs.guard_slots > 0)
-      pay = false;  // rows beside a 1D mesh: no kernel of their own
-    else if (!ctx->logsph)
+    if (!ctx->logsph)
       pay = ctx->prec == APT_PREC_FP64 ? f64_runs_pay(ctx->mesh.dim, kept, h[1])
                                        : mixed_runs_pay(ctx->mesh.dim, kept, h[1]);
   } else {

@@ -98,3 +98,37 @@ def test_log_spherical_mesh_with_guard_planes(precision):
     assert np.abs(out[0][0]).max() > 0
     for a, b in zip(*out):
         assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("precision", [apt.APT_PREC_FP64, apt.APT_PREC_MIXED])
+@pytest.mark.parametrize("N,guard", [((50,), [2, 2, 0]), ((50,), [2, 0, 1]), ((21, 18), [2, 2, 1])])
+def test_cartesian_mesh_with_idle_guards(N, guard, precision):
+    """Guard cells along axes that the mesh does not have: a sort changes nothing
+    but the order of the slots."""
+    c = Case(N, 5, theta=(0.1, 0.1), drift=(0.2, -0.2), Bbg=(0.3, 0.0, 1.0), data_interval=1)
+    dims = [c.N[q] + 2 * guard[q] for q in range(3)]
+    p = c.oracle().particles()
+    at = [p["cell"] % c.dims[0], p["cell"] // c.dims[0], np.full(c.nptc, guard[2])]
+    if len(N) == 1:
+        at[1] = at[1] + guard[1]
+    p["cell"] = (at[0] + dims[0] * (at[1] + dims[1] * at[2])).astype(np.uint32)
+    out = []
+    for sort in (False, True):
+        env = apt.sim_environment(apt.SimParams(
+            N=c.N, guard=guard, periodic_boundary=[True] * 3, max_ptc_number=c.nptc,
+            precision=precision, data_interval=1))
+        d = apt.sim_data(env)
+        rng = np.random.default_rng(4)
+        for which in (apt.FIELD_E, apt.FIELD_B):
+            for q in range(3):
+                d.set_field(which, q, rng.normal(size=env.ncell()))
+        d.set_particles(p)
+        if sort:
+            d.sort_particles()
+        pu = apt.ptc_updater(env)
+        for step in range(2):
+            pu.update_particles(d, 0.3 * c.dt, step)
+        out.append([d.get_field(apt.FIELD_J, q) for q in range(3)] +
+                   [np.sort(d.get_particles()["x1"])])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b, equal_nan=True)
